@@ -1576,39 +1576,45 @@ int launch_gemm(const GemmBatch& b_in, int aload, int blayout, bool a_relu,
     return post_layernorm(b, s);
   }
   // bf16 activations and weights: gemm_bf16.hip (what it does not take, outputs
-  // that its row stores cannot write, runs below)
-  if (bf16 && bf16_pipe_eligible(b, aload, a_relu) && b.ksplit <= 16) {
-    const bool can_split = splitk_eligible(b);
-    if (b.ksplit <= 1 ||
-        (can_split && b.g[0].K / 64 >= b.ksplit &&
-         (int64_t)b.ksplit * b.g[0].M * b.g[0].N * b.ngroups <= b.part_ws_elems)) {
-      int S = 1;
-      const int tile = plan_bf16_pipe(b, aload, can_split, &S);
-      b.ksplit = S;
-      int64_t items = 0;
-      double flops = 0.0, bytes = 0.0;
-      for (int i = 0; i < b.ngroups; ++i) {
-        const GemmArgs& g = b.g[i];
-        b.g[i].part = S > 1 ? b.part_ws + (int64_t)i * S * g.M * g.N : nullptr;
-        items = std::max(items, (int64_t)g.M * (g.N / 4));
-        flops += 2.0 * g.M * (double)g.N * g.K;
-        bytes += 2.0 * ((double)g.M * g.K + (double)g.N * g.K) +
-                 ((g.flags & EPI_BF16OUT) ? 2.0 : 4.0) * g.M * (double)g.N;
-      }
-      hipEvent_t ev = prof_start(s);
-      const int rc = launch_bf16_pipe(b, aload, tile, s);
-      if (rc) return rc;
-      if (S > 1) {
-        launch_reduce(b, dim3((unsigned)((items + 255) / 256), 1, b.ngroups), s);
-        GS_CHECK_HIP(hipGetLastError());
-      }
-      if (ev)
-        prof_stop(s, ev,
-                  gemm_prof_name(aload == A_CONV_H ? "gemm_bf16_pipe_kernel<A_CONV_H>"
-                                                   : "gemm_bf16_pipe_kernel<A_PLAIN_H>", b).c_str(),
-                  flops, bytes);
-      return post_layernorm(b, s);
+  // that its row stores cannot write, runs below). K is cut by the rule of the
+  // 128 x 128 kernel, and a rotation is rounded as that kernel or as the 256-row
+  // kernels do it, by the number of 256 x 128 tiles: the split and the rounding
+  // that such launches have always had, so that a model's bf16 results, in which
+  // the layers after one amplify its last bit, stay the same.
+  if (bf16 && bf16_pipe_eligible(b, aload, a_relu)) {
+    if (b.ksplit > 1)
+      GS_REQUIRE(splitk_eligible(b) && b.g[0].K / 64 >= b.ksplit &&
+                     (int64_t)b.ksplit * b.g[0].M * b.g[0].N * b.ngroups <= b.part_ws_elems,
+                 "gemm: requested split-K needs a K step per range and must fit the scratch");
+    else if (b.ksplit == 0)
+      b.ksplit = plan_ksplit(b, max_tiles);
+    const int S = b.ksplit;
+    int64_t items = 0, tiles256 = 0;
+    double flops = 0.0, bytes = 0.0;
+    for (int i = 0; i < b.ngroups; ++i) {
+      const GemmArgs& g = b.g[i];
+      b.g[i].part = S > 1 ? b.part_ws + (int64_t)i * S * g.M * g.N : nullptr;
+      items = std::max(items, (int64_t)g.M * (g.N / 4));
+      tiles256 += (int64_t)((g.M + 255) / 256) * ((g.N + 127) / 128);
+      flops += 2.0 * g.M * (double)g.N * g.K;
+      bytes += 2.0 * ((double)g.M * g.K + (double)g.N * g.K) +
+               ((g.flags & EPI_BF16OUT) ? 2.0 : 4.0) * g.M * (double)g.N;
     }
+    for (int i = 0; i < b.ngroups; ++i)
+      if ((b.g[i].flags & EPI_ROPE) && S == 1 && tiles256 < 512) b.g[i].flags |= EPI_ROPE_SEP;
+    hipEvent_t ev = prof_start(s);
+    const int rc = launch_bf16_pipe(b, aload, plan_bf16_pipe(b, aload), s);
+    if (rc) return rc;
+    if (S > 1) {
+      launch_reduce(b, dim3((unsigned)((items + 255) / 256), 1, b.ngroups), s);
+      GS_CHECK_HIP(hipGetLastError());
+    }
+    if (ev)
+      prof_stop(s, ev,
+                gemm_prof_name(aload == A_CONV_H ? "gemm_bf16_pipe_kernel<A_CONV_H>"
+                                                 : "gemm_bf16_pipe_kernel<A_PLAIN_H>", b).c_str(),
+                flops, bytes);
+    return post_layernorm(b, s);
   }
   // fp32 plain / concat rows with NT weights below one round of 256 x 128
   // tiles take the direct-to-LDS kernel, split by its own cost model

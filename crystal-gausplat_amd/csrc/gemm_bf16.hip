@@ -42,7 +42,6 @@ __device__ __forceinline__ void const_for(std::integer_sequence<int, I...>, F&& 
 //   16384 x 3072, K = 1024             122 -> 110
 //   24576 x 4096, K = 1024, GELU       284 -> 266
 //   12288 x 6144, K = 7168            1263 -> 1011 (1071 TFLOP/s)
-//   2048 x 1024, K = 1024, residual     30 -> 16
 // A 256 x 256 tile of four waves (128 x 128 each, one per SIMD) took 351 us at
 // 24576 x 4096 x 1024: nothing to run while its only wave waits.
 // Raised wave priority around the MFMAs: 256 x 256 tiles 3-5 % slower.
@@ -254,40 +253,23 @@ bool bf16_pipe_eligible(const GemmBatch& b, int aload, bool a_relu) {
   return true;
 }
 
-// Tile and K split of a launch: the tiles of a CU (between the mean and the busiest
-// CU's) times their time, a fixed 4 us, and for a split the partials' way through
-// the scratch (written, read and the output written, at 4 TB/s) and 3 us for its
-// launch; a launch that writes the next LayerNorm has it in that pass. Ranges keep
-// at least 256 of K.
-int plan_bf16_pipe(const GemmBatch& b, int aload, bool can_split, int* ksplit) {
-  const GemmArgs& g0 = b.g[0];
-  const int ks = pipe_deep(b, aload == A_CONV_H) ? 64 : 32, steps = g0.K / ks;
-  double mn = 0.0, best = 0.0;
-  for (int i = 0; i < b.ngroups; ++i) mn += (double)b.g[i].M * b.g[i].N;
+// Tile of a launch whose K is cut into b.ksplit ranges: the tiles of a CU (between
+// the mean and the busiest CU's) times their time.
+int plan_bf16_pipe(const GemmBatch& b, int aload) {
+  const int ks = pipe_deep(b, aload == A_CONV_H) ? 64 : 32, S = std::max(b.ksplit, 1);
+  const double k64 = (b.g[0].K / ks + S - 1) / S * ks / 64.0;
+  double best = 0.0;
   int tile = 0;
-  *ksplit = 1;
   for (int c = 0; c < kPipeNumTiles; ++c) {
     const PipeTile& t = kPipeTiles[c];
     int64_t tiles = 0;
     for (int i = 0; i < b.ngroups; ++i)
       tiles += (int64_t)((b.g[i].M + t.bm - 1) / t.bm) * ((b.g[i].N + t.bn - 1) / t.bn);
-    for (int S = 1; S <= 16; ++S) {
-      if (b.ksplit > 0 && S != b.ksplit) continue;
-      if (S > 1 && b.ksplit == 0 &&
-          (!can_split || g0.K / S < 256 || (double)S * mn > (double)b.part_ws_elems))
-        break;
-      const double mean = (double)tiles * S / kCUs, most = (double)((tiles * S + kCUs - 1) / kCUs);
-      const double k64 = (steps + S - 1) / S * ks / 64.0;
-      double cost = 4.0 + std::max(t.epi + k64 * t.lat, 0.5 * (mean + most) * (t.epi + k64 * t.thr));
-      if (S > 1)
-        cost += 3.0 + (2 * S + 1) * mn * 4.0 / 4e6;
-      else if (g0.flags & EPI_LNOUT)
-        cost += 3.0 + mn * 8.0 / 4e6;
-      if (best == 0.0 || cost < best) {
-        best = cost;
-        tile = c;
-        *ksplit = S;
-      }
+    const double mean = (double)tiles * S / kCUs, most = (double)((tiles * S + kCUs - 1) / kCUs);
+    const double cost = std::max(t.epi + k64 * t.lat, 0.5 * (mean + most) * (t.epi + k64 * t.thr));
+    if (c == 0 || cost < best) {
+      best = cost;
+      tile = c;
     }
   }
   return tile;

@@ -355,6 +355,12 @@ __device__ __forceinline__ void w2_epi_row(const GemmArgs& p, const floatx16& q0
   epi_store<false, NB>(p, flags, row0, col0, stage, lane);
 }
 
+// a * b + c in two roundings: the operation without a contraction into a multiply-add.
+__device__ __forceinline__ float mul_add_sep(float a, float b, float c) {
+#pragma clang fp contract(off)
+  return a * b + c;
+}
+
 // Row epilogue for accumulators of the transposed product (the weight fragment
 // as the MFMA's first operand): lane l32 holds row row0 + l32 and register
 // 4 g + j of q0 (q1) its column col0 (+ 32) + 8 g + 4 hl + j, so the stage is
@@ -402,10 +408,21 @@ __device__ __forceinline__ void w2_epi_row_t(const GemmArgs& p, const floatx16& 
           x0 = x0 + bv[g + 4][j];
           x1 = x1 + bv[g + 6][j];
         }
-        r[0][j] = y0 * cy[g][j] - y1 * sy[g][j];
-        r[1][j] = y1 * cy[g][j] + y0 * sy[g][j];
-        r[2][j] = x0 * cx[g][j] - x1 * sx[g][j];
-        r[3][j] = x1 * cx[g][j] + x0 * sx[g][j];
+        // the rounding of w2_epi_row (the sine product rounded, the cosine's in the
+        // multiply-add), or with EPI_ROPE_SEP that of gemm_epilogue_t (both rounded)
+        const float s0 = -(y1 * sy[g][j]), s1 = y0 * sy[g][j];
+        const float s2 = -(x1 * sx[g][j]), s3 = x0 * sx[g][j];
+        if (flags & EPI_ROPE_SEP) {
+          r[0][j] = mul_add_sep(y0, cy[g][j], s0);
+          r[1][j] = mul_add_sep(y1, cy[g][j], s1);
+          r[2][j] = mul_add_sep(x0, cx[g][j], s2);
+          r[3][j] = mul_add_sep(x1, cx[g][j], s3);
+        } else {
+          r[0][j] = __builtin_fmaf(y0, cy[g][j], s0);
+          r[1][j] = __builtin_fmaf(y1, cy[g][j], s1);
+          r[2][j] = __builtin_fmaf(x0, cx[g][j], s2);
+          r[3][j] = __builtin_fmaf(x1, cx[g][j], s3);
+        }
       }
 #pragma unroll
       for (int h = 0; h < 4; ++h)

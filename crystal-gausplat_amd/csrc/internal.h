@@ -81,6 +81,7 @@ enum EpiFlags : int {
   EPI_BF16OUT = 256, // C holds bf16 (ldc in elements; with SCATTER the scattered store); not with DUAL
   EPI_LNOUT = 512,   // also the LayerNorm of every output row into lnout (see GemmArgs)
   EPI_DUAL_RELU_H = 1024,  // with EPI_DUAL: C2 holds bf16 and receives bf16(max(v, 0))
+  EPI_ROPE_SEP = 2048,     // with EPI_ROPE: both products of the rotation rounded (set by launch_gemm)
 };
 
 struct GemmArgs {
@@ -177,7 +178,7 @@ int plan_h3(const GemmBatch& b, bool can_split, int* ksplit);  // the tile, and 
 // GEMM / conv with bf16 A and bf16 NT weights (gemm_bf16.hip)
 bool bf16_pipe_eligible(const GemmBatch& b, int aload, bool a_relu);
 int launch_bf16_pipe(const GemmBatch& b, int aload, int tile, hipStream_t s);
-int plan_bf16_pipe(const GemmBatch& b, int aload, bool can_split, int* ksplit);
+int plan_bf16_pipe(const GemmBatch& b, int aload);  // the tile, for b.ksplit ranges of K
 // Split planes and powers of two of `rows` weight rows of K values (K % 32 == 0).
 int launch_split_rows(const float* in, int64_t rows, int32_t K, float* out, int32_t* bexp,
                       int64_t bexp_ld, hipStream_t s);
