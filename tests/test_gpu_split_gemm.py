@@ -89,6 +89,15 @@ def test_linear_split_row_and_column_magnitudes():
     assert_bound(linear(x, w), x, w, extra=2.0 ** -140)
 
 
+@pytest.mark.parametrize("xs,ws", [(1e-36, 1e35), (1e-20, 1e33), (1e-30, 1e35), (1e-4, 1e34), (1e30, 1e-36)])
+def test_linear_split_magnitudes_that_cancel(xs, ws):
+    """Rows of x and of W that only together are in range."""
+    case(f"split linear magnitudes {xs} {ws}")
+    M, K, N = 2560, 1024, 512
+    x, w = rnd(M, K) * np.float32(xs), rnd(N, K) * np.float32(ws)
+    assert_bound(linear(x, w), x, w, extra=2.0 ** -140)
+
+
 def test_linear_split_wide_rows():
     """One element 2^26 times the others, met by a zero weight: the others keep
     full precision (their products are all the result)."""
