@@ -1554,7 +1554,7 @@ int launch_gemm(const GemmBatch& b_in, int aload, int blayout, bool a_relu,
   // smaller error; what it does not take runs below)
   if (!bf16 && blayout == B_NT && b.kernel == 0 && h3_eligible(b, aload, a_relu)) {
     int S = 1;
-    const int tile = plan_h3(b, splitk_eligible(b), &S);
+    const int tile = plan_h3(b, aload, splitk_eligible(b), &S);
     b.ksplit = S;
     int64_t items = 0;
     double flops = 0.0, bytes = 0.0;

@@ -85,6 +85,14 @@ __device__ __forceinline__ void lds_dma16(const float* gptr, uint32_t lds) {
                : "memory", "m0");
 }
 
+// The same from a wave-uniform base and a lane's 32-bit byte offset.
+__device__ __forceinline__ void lds_dma16_off(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds), "v"(off), "s"(base)
+               : "memory", "m0");
+}
+
 constexpr int W2M = 256, W2N = 128, W2K = 32;
 
 constexpr int W2_SS = 68;                    // epilogue stage row stride (floats)

@@ -174,7 +174,7 @@ int check_gemm(const GemmArgs& a, int aload, int blayout, bool bf16 = false);
 constexpr int kH3MinK = 128;
 bool h3_eligible(const GemmBatch& b, int aload, bool a_relu);
 int launch_gemm_h3(const GemmBatch& b, int aload, bool a_relu, int tile, hipStream_t s);
-int plan_h3(const GemmBatch& b, bool can_split, int* ksplit);  // the tile, and the K split
+int plan_h3(const GemmBatch& b, int aload, bool can_split, int* ksplit);  // the tile, and the K split
 // GEMM / conv with bf16 A and bf16 NT weights (gemm_bf16.hip)
 bool bf16_pipe_eligible(const GemmBatch& b, int aload, bool a_relu);
 int launch_bf16_pipe(const GemmBatch& b, int aload, int tile, hipStream_t s);

@@ -5,8 +5,9 @@ the range that two fp16 terms cover, against 64-bit products.
 Bound per element: every product term is exact in the fp32 accumulation, which
 takes at most 3 K / 16 + 32 roundings (each of at most 2^-23 of a partial sum, and
 those are at most S = sum |x w|), and the dropped parts of the operands are below
-2^-21 S together: |error| <= (3 K / 16 + 32) 2^-23 S + 2^-21 S. Values smaller than
-2^-29 of their row's largest magnitude keep an absolute 2^-50 of it, also covered."""
+2^-21 S together: |error| <= (3 K / 16 + 32) 2^-23 S + 2^-21 S. What small values lose
+beside large ones is below 1.5 2^-21 S where the sums certify it, and such elements
+are computed in fp32 where they do not."""
 import numpy as np
 import pytest
 import torch
@@ -107,6 +108,66 @@ def test_linear_split_wide_rows():
     x[:, 7] = 2.0 ** 26
     w[:, 7] = 0.0
     assert_bound(linear(x, w), x, w)
+
+
+def assert_wide(got, x, w):
+    """assert_bound, and the errors of all elements together within 1.5e-6 of S
+    (three roundings of 2^-24 per 512 of K and the kernel's 1.5 2^-21)."""
+    assert_bound(got, x, w)
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    S = np.abs(x64) @ np.abs(w64).T
+    assert np.sqrt(np.mean(((got - x64 @ w64.T) / S) ** 2)) < 1.5e-6
+
+
+@pytest.mark.parametrize("M,K,N", [(2560, 512, 1024), (1100, 2048, 644)])
+@pytest.mark.parametrize("loud,rest", [(2.0 ** -7, -22), (2.0 ** -7, -45), (1.0, -20), (1.0, -26), (1.0, -37),
+                                       (32.0, -30), (2.0 ** 26, -5), (2.0 ** 26, -30)])
+def test_linear_split_one_loud_value(loud, rest, M, K, N):
+    """A loud value that meets zeros: the others' products are all the result,
+    whatever the two magnitudes; in x, in W, and behind the sampled values."""
+    case(f"split linear loud {loud} rest 2^{rest} M={M}")
+    for at in (7, K - 3):
+        x, w = rnd(M, K, scale=2.0 ** rest), rnd(N, K)
+        x[:, at], w[:, at] = loud, 0.0
+        assert_wide(linear(x, w), x, w)
+    x, w = rnd(M, K), rnd(N, K, scale=2.0 ** rest)
+    x[:, 7], w[:, 7] = 0.0, loud
+    assert_wide(linear(x, w), x, w)
+
+
+def test_linear_split_values_of_all_magnitudes():
+    """Rows whose values spread over 2^-60 .. 1, and rows of zeros."""
+    case("split linear spread")
+    M, K, N = 2560, 512, 1024
+    x = rnd(M, K) * np.exp2(RNG.uniform(-60, 0, (M, K))).astype(np.float32)
+    w = rnd(N, K) * np.exp2(RNG.uniform(-60, 0, (N, K))).astype(np.float32)
+    x[5::7, :] = 0.0
+    w[3::11, :] = 0.0
+    x[2, :300] = 0.0
+    got = linear(x, w)
+    assert_bound(got, x, w)
+    assert not got[5::7].any() and not got[:, 3::11].any()
+
+
+def test_conv_split_one_loud_channel():
+    """A loud input channel with zero weights, the others far below it, also where
+    the window's first taps are outside the image."""
+    case("split conv loud channel")
+    B, H, W, Ci, Co = 2, 40, 64, 96, 256
+    x, w = rnd(B, H, W, Ci, scale=1e-9), rnd(Co, 3, 3, Ci, scale=0.05)
+    x[..., 50], w[..., 50] = 3.0, 0.0
+    conv = lambda a, f: torch.nn.functional.conv2d(
+        torch.from_numpy(a.astype(np.float64)).permute(0, 3, 1, 2),
+        torch.from_numpy(f.astype(np.float64)).permute(0, 3, 1, 2), padding=1).permute(0, 2, 3, 1).numpy()
+    for relu in (False, True):
+        xi = np.maximum(x, 0) if relu else x
+        ref, S = conv(xi, w), conv(np.abs(xi), np.abs(w))
+        y = empty(B, H, W, Co)
+        xd, wd = dev(x), dev(w)
+        G.check(G.lib().gs_hip_conv2d(G.ptr(xd), B, H, W, Ci, G.ptr(wd), None, G.ptr(y), Co, 3, 1, 1, 1,
+                                      G.CONV_RELU_IN if relu else 0, None, stream()))
+        K = 9 * Ci
+        assert (np.abs(host(y) - ref) <= ((3 * K / 16 + 32) * 2.0 ** -23 + 2.0 ** -21) * S).all()
 
 
 def test_linear_split_rows_do_not_depend_on_their_tile():
