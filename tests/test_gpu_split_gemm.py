@@ -270,14 +270,14 @@ def test_context_weights_follow_set_weight(tiny_cfg):
 
 
 # ---- attention on fp16 split products --------------------------------------------
-def attention(q, k, v):
+def attention(q, k, v, prec=0):
     B, Nq, D = q.shape
     Nkv, H = k.shape[1], D // 64
     o = empty(B, Nq, D)
     qd, kd, vd = dev(q), dev(k), dev(v)
     sq, sk = (Nq * D, 64, D), (Nkv * D, 64, D)
-    G.check(G.lib().gs_hip_attention(G.ptr(qd), G.ptr(kd), G.ptr(vd), G.ptr(o), B, H, Nq, Nkv, 64, 0.125,
-                                     *sq, *sk, *sk, *sq, stream()))
+    G.check(G.lib().gs_hip_attention_prec(G.ptr(qd), G.ptr(kd), G.ptr(vd), G.ptr(o), B, H, Nq, Nkv, 64, 0.125,
+                                          *sq, *sk, *sk, *sq, prec, stream()))
     return host(o)
 
 
@@ -316,6 +316,69 @@ def test_attention_split_magnitudes(qs, ks, vs, B, Nkv):
     q, k, v = rnd(B, 200, 768, scale=qs), rnd(B, Nkv, 768, scale=ks), rnd(B, Nkv, 768, scale=vs)
     ref, bound = attention64(q, k, v)
     assert (np.abs(attention(q, k, v) - ref) <= bound + 1e-44).all()
+
+
+def check_attention(q, k, v, factor=1.0, prec=0):
+    """Against 64 bits with attention64's bound, and with small inputs together within
+    1.5e-6 of sum p |v| (factor: what large scores allow besides)."""
+    ref, bound = attention64(q, k, v)
+    err = np.abs(attention(q, k, v, prec) - ref)
+    assert (err <= bound).all()
+    B, Nq, D = q.shape
+    h = lambda t: t.astype(np.float64).reshape(B, -1, D // 64, 64).transpose(0, 2, 1, 3)
+    s = h(q) @ h(k).transpose(0, 1, 3, 2) * 0.125
+    p = np.exp(s - s.max(-1, keepdims=True))
+    S = ((p / p.sum(-1, keepdims=True)) @ np.abs(h(v))).transpose(0, 2, 1, 3).reshape(B, Nq, D)
+    S = np.where(S > 0, S, 1.0)
+    assert np.sqrt(np.mean((err / S) ** 2)) < 1.5e-6 * factor
+
+
+@pytest.mark.parametrize("prec", [0, 2])
+@pytest.mark.parametrize("qs,ks,vs", [(4e5, 1e-5, 1.0), (1e8, 1e-8, 1.0), (1e12, 1e-12, 1.0), (1e-12, 1e12, 1.0),
+                                      (1e-30, 1e30, 1e-30), (1.0, 1.0, 1e30)])
+@pytest.mark.parametrize("B,Nkv", [(1, 700), (20, 200)])
+def test_attention_split_magnitudes_that_cancel(qs, ks, vs, B, Nkv, prec):
+    """Large queries with small keys and the reverse: scores of order 1."""
+    case(f"split attention scales {qs} {ks} {vs} B={B} precision {prec}")
+    q, k, v = rnd(B, 200, 768, scale=qs), rnd(B, Nkv, 768, scale=ks), rnd(B, Nkv, 768, scale=vs)
+    check_attention(q, k, v, prec=prec)
+
+
+@pytest.mark.parametrize("loud", [30.0, 1e6, 1e12])
+@pytest.mark.parametrize("B,Nkv", [(1, 700), (20, 200)])
+def test_attention_split_loud_values(loud, B, Nkv):
+    """Loud values beside small ones that are all the result: a head dimension of Q
+    that meets zeros in K (and the reverse), one dimension of V, one key of V
+    without probability."""
+    case(f"split attention loud {loud} B={B}")
+    q, k, v = rnd(B, 200, 768), rnd(B, Nkv, 768), rnd(B, Nkv, 768)
+    for t, z in ((q, k), (k, q)):
+        a, b = t.copy(), z.copy()
+        a[..., 9::64], b[..., 9::64] = loud, 0.0
+        check_attention(*((a, b, v) if t is q else (b, a, v)))
+    small = v / np.float32(loud)
+    small[..., 5::64] = rnd(B, Nkv, 12)  # the other dimensions are small beside it
+    check_attention(q, k, small)
+    small = v / np.float32(loud)
+    small[:, 33] *= np.float32(loud)
+    k2, q2 = k.copy(), q.copy()
+    q2[..., 2::64] = 40.0
+    k2[..., 2::64] = 0.0
+    k2[:, 33, 2::64] = -60.0  # a score of -300: its large V does not count
+    check_attention(q2, k2, small, 4.0)
+
+
+@pytest.mark.parametrize("below", [10, 17, 24, 30, 40, 60])
+@pytest.mark.parametrize("B,Nkv", [(1, 700), (20, 200)])
+def test_attention_split_sink(below, B, Nkv):
+    """One key takes nearly all weight and has a V of zeros: the result is that of
+    the others, 2^-below of its weight each."""
+    case(f"split attention sink 2^-{below} B={B}")
+    q, k, v = rnd(B, 200, 768, scale=0.3), rnd(B, Nkv, 768, scale=0.3), rnd(B, Nkv, 768)
+    q[..., 2::64], k[..., 2::64] = 4.0, 0.0
+    k[:, Nkv // 2, 2::64] = below * np.log(2) * 8 / 4.0
+    v[:, Nkv // 2] = 0.0
+    check_attention(q, k, v, 4.0)
 
 
 @pytest.mark.parametrize("B,Nkv", [(1, 700), (20, 200)])
