@@ -454,12 +454,14 @@ __device__ __attribute__((aligned(64))) float g_zero16[16] = {};
 bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15) == 0; }
 
 // The staged epilogue of the one-wave-per-SIMD kernels stores 4 columns per
-// lane with vector accesses.
+// lane with vector accesses, at 32-bit byte offsets within a block of 32 rows
+// (kRowEpiMaxLdc).
 bool row_epi_ok(const GemmArgs& g) {
   if (g.flags & EPI_SCATTER)  // 4-column segments stay within one output pixel
     return g.sc_C % 4 == 0 && g.sc_Cout % 4 == 0 && g.N % 4 == 0 && aligned16(g.C) &&
            !(g.flags & (EPI_RES1 | EPI_RES2 | EPI_ROPE | EPI_DUAL));
   if (g.N % 4 || g.ldc % 4 || !aligned16(g.C)) return false;
+  if (g.ldc > kRowEpiMaxLdc) return false;
   if ((g.flags & EPI_RES1) && (g.ldr1 % 4 || !aligned16(g.R1))) return false;
   if ((g.flags & EPI_RES2) && (g.ldr2 % 4 || !aligned16(g.R2))) return false;
   if ((g.flags & EPI_DUAL) && !aligned16(g.C2)) return false;

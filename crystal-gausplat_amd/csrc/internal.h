@@ -166,12 +166,15 @@ struct GemmBatch {
 int launch_gemm(const GemmBatch& b, int aload, int blayout, bool a_relu,
                 hipStream_t s, bool bf16 = false);
 int check_gemm(const GemmArgs& a, int aload, int blayout, bool bf16 = false);
+// Longest output rows (floats) that the staged row epilogue takes: 32 of them at
+// 32-bit byte offsets. Wider outputs run on the kernels that store with 64.
+constexpr int64_t kRowEpiMaxLdc = ((int64_t)1 << 32) / (32 * 4) - 1;
 
 // fp32 GEMM through two-term fp16 splits (gemm_h3.hip): plain, concat and conv
 // (with or without ReLU prologue) A, NT B with split planes, K >= kH3MinK, the
 // row epilogue. tile indexes the launcher's tile table; b.ksplit > 1 writes
 // partials for the split-K reduce.
-constexpr int kH3MinK = 128;
+constexpr int kH3MinK = 128, kH3MaxRow = 1 << 22;  // K, and the longest row it takes
 bool h3_eligible(const GemmBatch& b, int aload, bool a_relu);
 int launch_gemm_h3(const GemmBatch& b, int aload, bool a_relu, int tile, hipStream_t s);
 int plan_h3(const GemmBatch& b, int aload, bool can_split, int* ksplit);  // the tile, and the K split
