@@ -10,11 +10,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-template <class F, int... I>
-__device__ __forceinline__ void const_for(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>()), ...);
-}
-
 // Workgroup tile BM x BN of WVM x WVN waves, each (BM / WVM) x (BN / WVN) in MFMA
 // 32x32x16 blocks; KS-deep K steps streamed straight into one of NST LDS stages
 // (global_load_lds_dwordx4).

@@ -1,7 +1,10 @@
-// Device pieces shared by the GEMM kernels (gemm.hip, gemm_h3.hip): activation
+// Device pieces shared by the GEMM kernels: activation
 // functions, split-K ranges, direct-to-LDS loads and the staged row epilogue.
 #pragma once
 #include <stdint.h>
+
+#include <type_traits>
+#include <utility>
 
 #include "internal.h"
 
@@ -11,6 +14,12 @@ namespace gs {
 namespace {
 
 constexpr int GROUP_M = 8;
+
+// f(0), f(1), ... with the index as a constant.
+template <class F, int... I>
+__device__ __forceinline__ void const_for(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>()), ...);
+}
 
 // GELU, tanh form (src/nn/vit.cr:130-148): 0.5*v*(1 + tanh(u)) with
 // u = c*(v + 0.044715*v^3), c = (float)sqrt(2/pi). Evaluated through the exact

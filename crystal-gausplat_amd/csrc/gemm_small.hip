@@ -145,7 +145,7 @@ int launch_linear_small(const GemmArgs& a, int prec, hipStream_t s) {
              "linear_small: bad arguments");
   const dim3 grid((unsigned)(((a.M + 31) / 32) * ((a.N + 31) / 32)));
   hipEvent_t ev = prof_start(s);
-  // waves: four to eight steps of K each
+  // waves: at most eight steps of K each
 #define GS_SMALL(NW, P) hipLaunchKernelGGL((linear_small_kernel<NW, P>), grid, dim3(64 * NW), 0, s, a)
 #define GS_SMALL_NW(P)      \
   if (a.K <= 256)           \
