@@ -129,8 +129,12 @@ void gs_seed_uniform(uint64_t seed, const char* name, float lo, float hi,
  * on them directly; other shapes on zero-padded copies of x and W in
  * stream-ordered scratch (allocated and released on `stream`). Larger fp32
  * calls (w_layout 0) multiply two-term fp16 splits of both operands on the fp16
- * matrix cores (fp32 accumulate; closer to the fp64 product than fp32 MFMA,
- * any magnitude, infinities and NaN as in fp32), others run on fp32 MFMA.
+ * matrix cores, with the split weight in such scratch (4 bytes per value). Each
+ * operand keeps 22 to 24 significand bits; with fp32 accumulation the result is
+ * closer to the fp64 product than fp32 MFMA's on ordinary operands, and what
+ * values far below their row's largest lose is below 2^-20 of the element's sum
+ * of |x w| (elements for which that is not certain, and those that infinities
+ * or NaN reach, are computed in fp32). Others run on fp32 MFMA.
  * b, residual nullable. residual may alias y. */
 int32_t gs_hip_linear(const float* x, const float* w, const float* b, float* y,
                       int64_t M, int32_t K, int32_t N, int32_t w_layout,
@@ -166,11 +170,16 @@ int32_t gs_hip_attention(const float* q, const float* k, const float* v,
 
 /* gs_hip_attention with a choice of arithmetic, as gs_hip_linear's epilogue
  * flags choose it for the linears: precision 0 = fp32 (gs_hip_attention itself:
- * two-term fp16 splits of the operands on the fp16 matrix cores, closer to the
- * fp64 result than fp32 MFMA, any magnitude, infinities and NaN as in fp32); 1 = the bf16-input / fp32-accumulate variant (q, k, v and the
- * softmax probabilities rounded to bf16); 2 = fp32 through bf16x6 split products (fp32-level accuracy;
- * launches that split the keys run precision 0's kernel). Precisions 1 and 2 need
- * head_dim 64 and 16-byte aligned rows. */
+ * two-term fp16 splits of q, k, v and the probabilities, 22 to 24 significand bits
+ * each, on the fp16 matrix cores; closer to the fp64 result than fp32 MFMA on
+ * ordinary operands; queries with an output for which the split's loss is not
+ * certain to be below 2^-20 of its sum of p |v|, and those that infinities or NaN
+ * reach, are computed in fp32); 1 = the bf16-input / fp32-accumulate variant
+ * (q, k, v and the softmax probabilities rounded to bf16); 2 = fp32 through bf16x6
+ * split products (exact three-term splits), except that launches of fewer than
+ * three workgroups of 128 queries per compute unit run precision 0's kernel
+ * (their error against fp64 is smaller there). Precisions 1 and 2 need head_dim 64
+ * and 16-byte aligned rows. */
 int32_t gs_hip_attention_prec(const float* q, const float* k, const float* v,
                               float* o, int32_t B, int32_t H, int32_t Nq,
                               int32_t Nkv, int32_t head_dim, float scale,
@@ -296,7 +305,9 @@ typedef struct gs_mastr_config {
   int32_t precision;     /* 0 = fp32 (GEMMs and convolutions with K >= 128 as
                             products of two-term fp16 splits of both operands,
                             fp32 accumulate, error vs fp64 below the fp32
-                            MFMA kernels'; the rest on fp32 MFMA);
+                            MFMA kernels' on ordinary operands, see
+                            gs_hip_linear; the context holds the weights a
+                            second time, split; the rest on fp32 MFMA);
                             1 = bf16-input / fp32-accumulate
                             MFMA GEMMs and attention (linear_layout 0 only);
                             2 = fp32 GEMMs and convolutions on bf16 matrix
