@@ -368,6 +368,19 @@ def test_attention_split_loud_values(loud, B, Nkv):
     check_attention(q2, k2, small, 4.0)
 
 
+@pytest.mark.parametrize("B,Nkv", [(1, 700), (20, 200)])
+def test_attention_split_zero_dimensions(B, Nkv):
+    """Heads narrower than 64, padded with zeros, and a head of zeros."""
+    case(f"split attention zero dimensions B={B}")
+    q, k, v = rnd(B, 200, 768), rnd(B, Nkv, 768), rnd(B, Nkv, 768)
+    for t in (q, k, v):
+        t.reshape(B, -1, 12, 64)[..., 40:] = 0.0
+    v[..., 64:128] = 0.0
+    check_attention(q, k, v)
+    got = attention(q, k, v).reshape(B, 200, 12, 64)
+    assert not got[..., 40:].any() and not got[:, :, 1].any()
+
+
 @pytest.mark.parametrize("below", [10, 17, 24, 30, 40, 60])
 @pytest.mark.parametrize("B,Nkv", [(1, 700), (20, 200)])
 def test_attention_split_sink(below, B, Nkv):
