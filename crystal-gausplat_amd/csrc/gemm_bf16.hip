@@ -14,8 +14,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // 32x32x16 blocks; KS-deep K steps streamed straight into one of NST LDS stages
 // (global_load_lds_dwordx4).
 //
-// The matrix cores bound it, in practice the clock that their power leaves
-// (1.5-1.9 GHz) and what keeps them waiting. So:
+// What keeps the matrix cores waiting bounds it: at 24576 x 4096 x 1024 they are
+// busy 41 % of the time at 2.05 GHz, and waves wait 43-46 % of their cycles. So:
 // - One barrier per K step. A wave passes it with the last fragments of step k in
 //   registers, and with all its reads of that stage done: the stage is refilled
 //   with step k + NST at once, and step k + 1's first fragments are read under the
@@ -33,10 +33,11 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // slices, so all tiles give the same bits unless K is split.
 // Against the 256 x 128 kernel with two barriers per 32-deep step and the
 // register-staged 128 x 128 kernel (split in K for small launches) it replaces, us:
-//   16384 x 1024, K = 4096, residual   183 -> 144 (957 TFLOP/s)
-//   16384 x 3072, K = 1024             122 -> 110
-//   24576 x 4096, K = 1024, GELU       284 -> 266
-//   12288 x 6144, K = 7168            1263 -> 1011 (1071 TFLOP/s)
+//   16384 x 1024, K = 4096, residual   183 -> 138 (996 TFLOP/s)
+//   16384 x 3072, K = 1024             127 -> 113
+//   24576 x 4096, K = 1024, GELU       255 -> 232
+//   12288 x 6144, K = 7168            1198 -> 960 (1127 TFLOP/s)
+//   2048 x 1024, K = 1024, residual   25.6 -> 26.3 (same split of K)
 // A 256 x 256 tile of four waves (128 x 128 each, one per SIMD) took 351 us at
 // 24576 x 4096 x 1024: nothing to run while its only wave waits.
 // Raised wave priority around the MFMAs: 256 x 256 tiles 3-5 % slower.

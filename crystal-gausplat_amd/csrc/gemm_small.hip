@@ -7,8 +7,8 @@
 // loads in flight), multiplies them in the call's arithmetic, and the waves' sums are
 // added in wave order through LDS before the epilogue. So there is one launch and no
 // scratch: no split-K reduce pass, no bf16 copies of the operands.
-// M x K x N, before and after, a call in a stream of calls: fp32 256 x 512 x 256 19.6 ->
-// 7.2 us, 32 x 1024 x 4096 24.4 -> 11.5, 512 x 1024 x 1024 25.2 -> 20.1; bf16 256 x 512 x 256
+// M x K x N, before and after, a call in a stream of calls: fp32 256 x 512 x 256 24.1 ->
+// 7.7 us, 32 x 1024 x 4096 24.4 -> 11.5, 512 x 1024 x 1024 25.2 -> 20.1; bf16 256 x 512 x 256
 // 31.4 -> 6.8, bf16x6 23.6 -> 7.0. A fragment load touches 32 rows for 32 bytes each, so
 // long K is bound by the cache's tag rate: 256 x 2048 x 512 23.2 -> 18-20 us, but K = 4096
 // lost (27 -> 33), and more tiles or longer K stay on the LDS-staged kernels.
